@@ -274,4 +274,128 @@ template <> struct MF16<float> {
   __device__ __forceinline__ static frag scale(frag v, const float w[WN]) { return v * w[0]; }
 };
 
+// ---- float32 contractions on the bf16 matrix cores.  A float32 value is the exact sum
+// of three bf16 parts, hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid (24 bits in
+// three times 8, each rounded to nearest), and a product of two such sums keeps the six
+// part products down to 2^-16 of the leading one; the three dropped are at most 2^-24 of
+// it and of random sign, below the rounding of a float32 product.  Accumulation is
+// float32.  gfx950 runs bf16 MFMA at 16 times its float32 rate, so six products take
+// 3/8 of the float32 instructions' time.  An infinity's parts are inf - inf, so a
+// non-finite operand gives NaN where the float32 product might have kept an infinity.
+struct Parts8 {
+  bf16x8 h, m, l;
+};
+// The parts of two values, each pair packed (two conversions, two unpacks and two
+// subtractions per part).
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = __builtin_bit_cast(uint32_t, (bf16x2){(bf16)x0, (bf16)x1});
+  const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+  m = __builtin_bit_cast(uint32_t, (bf16x2){(bf16)r0, (bf16)r1});
+  l = __builtin_bit_cast(uint32_t, (bf16x2){(bf16)(r0 - __uint_as_float(m << 16)),
+                                            (bf16)(r1 - __uint_as_float(m & 0xffff0000u))});
+}
+__device__ __forceinline__ Parts8 split8(const float x[8]) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) split2(x[2 * j], x[2 * j + 1], h[j], m[j], l[j]);
+  Parts8 s;
+  s.h = __builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3]));
+  s.m = __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]));
+  s.l = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
+  return s;
+}
+// NT independent products side by side: A[i] B[i] added to lo[i] (the five small products)
+// and hi[i] (the leading one), which may be the same accumulator.
+template <int NT>
+__device__ __forceinline__ void mma_parts(const Parts8 (&a)[NT], const Parts8 (&b)[NT], f32x4* hi, f32x4* lo) {
+#define M3_STEP(acc, x, y) \
+  _Pragma("unroll") for (int i = 0; i < NT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i].x, b[i].y, acc[i], 0, 0, 0);
+  M3_STEP(lo, m, m)
+  M3_STEP(hi, h, h)
+  M3_STEP(lo, h, l)
+  M3_STEP(lo, l, h)
+  M3_STEP(lo, h, m)
+  M3_STEP(lo, m, h)
+#undef M3_STEP
+}
+
+// A [token][n] tile of N columns as three bf16 planes of CS rows of N / 8 16-byte slots.
+// Two orders of the columns in a row:
+//  * PAIRED: slot s holds the columns 32 (s / 4) + 4 (s % 4) + {0..3} and + {16..19}, the
+//    rows of a pair of state tiles that one lane of their accumulators holds, so that a
+//    32-wide step of a contraction over n with the state is one 16-byte read;
+//  * natural, for a tile that is also read transposed (col): 16 consecutive columns are
+//    two whole slots, so that a transposed read touches every bank (PAIRED they would be
+//    halves of four slots, on half of the banks: that took 40% of the LDS cycles of the
+//    float32 scan).
+// Slots are exchanged within a row by swz(row): 16 rows' reads of one slot, and the 8
+// rows of a transposed read's two, lie on different banks.
+template <int CS, int N, bool PAIRED>
+struct PlaneTile {
+  static constexpr int S = N / 8;                  // slots per row: 16, 8 or 4
+  uint4 p[3][CS * S];
+  __device__ __forceinline__ static int swz(int t) {
+    if constexpr (PAIRED) return (t >> (S == 16 ? 0 : S == 8 ? 1 : 2)) & (S - 1);
+    if constexpr (S == 16) return ((t >> 2) & 1) | ((t & 3) << 1) | (t & 8);
+    if constexpr (S == 8) return ((t >> 2) & 1) | (t & 2) | ((t >> 1) & 4);
+    return ((t >> 2) & 1) | ((t >> 2) & 2);
+  }
+  // the slot of columns 4 gi .. 4 gi + 3, and which half of it
+  __device__ __forceinline__ static int slot4(int gi) { return PAIRED ? 4 * (gi >> 3) + (gi & 3) : gi >> 1; }
+  __device__ __forceinline__ static int half4(int gi) { return PAIRED ? (gi >> 2) & 1 : gi & 1; }
+  // their offset in row t, in 8-byte units
+  __device__ __forceinline__ static int off4(int t, int gi) {
+    return 2 * (t * S + (slot4(gi) ^ swz(t))) + half4(gi);
+  }
+  __device__ __forceinline__ void put4(int t, int gi, const float x[4]) {
+    uint2 h, m, l;
+    split2(x[0], x[1], h.x, m.x, l.x);
+    split2(x[2], x[3], h.y, m.y, l.y);
+    const int o = off4(t, gi);
+    reinterpret_cast<uint2*>(p[0])[o] = h;
+    reinterpret_cast<uint2*>(p[1])[o] = m;
+    reinterpret_cast<uint2*>(p[2])[o] = l;
+  }
+  // operand of a contraction over n: row row0 + lane%16, the columns 32 q + 4 (lane/16) +
+  // {0..3} and + {16..19} of step q
+  __device__ __forceinline__ Parts8 row(int row0, int q, int lane) const {
+    const int t = row0 + (lane & 15), g = lane >> 4;
+    Parts8 f;
+    bf16x8* out[3] = {&f.h, &f.m, &f.l};
+    if constexpr (PAIRED) {
+      const int o = t * S + ((4 * q + g) ^ swz(t));
+#pragma unroll
+      for (int k = 0; k < 3; ++k) *out[k] = *reinterpret_cast<const bf16x8*>(&p[k][o]);
+    } else {
+      const int o0 = off4(t, 8 * q + g), o1 = off4(t, 8 * q + 4 + g);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const uint2 a = reinterpret_cast<const uint2*>(p[k])[o0], b = reinterpret_cast<const uint2*>(p[k])[o1];
+        *out[k] = __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
+      }
+    }
+    return f;
+  }
+  // operand of a contraction over tokens t0 + 8 (lane/16) + 0..7: column 16 nb + lane%16
+  __device__ __forceinline__ Parts8 col(int t0, int nb, int lane) const {
+    static_assert(!PAIRED, "natural order");
+    const int l = lane & 15, t = t0 + 8 * (lane >> 4) + (l >> 2), gi = 4 * nb + (l & 3);
+    const int o0 = off4(t, gi), o1 = off4(t + 4, gi);
+    Parts8 f;
+    bf16x8* out[3] = {&f.h, &f.m, &f.l};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const bf16x4* b = reinterpret_cast<const bf16x4*>(p[k]);
+      const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(b + o0));
+      const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(b + o1));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        (*out[k])[j] = lo[j];
+        (*out[k])[4 + j] = hi[j];
+      }
+    }
+    return f;
+  }
+};
+
 }  // namespace m3

@@ -3,19 +3,24 @@
 // The same operator as m3_scan_chunked.hip (the reference's mamba3_ssd_chunked_jax,
 // phases 1-7, src/base_model/models/mamba3_jax.py:327-419), for the float32
 // inputs the model hands its scan (mamba3.py:363-367 casts x, z, B and C to float32
-// before mamba3_siso_triton), with float32 MFMA operands (v_mfma_f32_16x16x4_f32,
-// float32 accumulation: exact float32 contractions) and 32-token chunks.
+// before mamba3_siso_triton), with float32 accuracy and 32-token chunks.
 //
-// The work is split differently from the bf16 kernel because a float32 MFMA costs
-// 16 times a bf16 one per FLOP, so the matrix work must be spread over every SIMD:
-// one workgroup of 12 waves per (batch, head) walks the chunks in order.  Output
-// waves 0-2 each own one (query block, key block) item of Y_diag (an S^T block, the
-// causal mask or the decay, M V over its keys), so three of the four SIMDs share it.
-// State waves 4-7 each own 16 columns of the value dimension (a p-tile): h^T[:, p-tile]
-// (all N rows) as 16x16 accumulators, that p-tile's Y_off = Q_r h^T and its state
-// update.  Auxiliary waves 8-11 take the larger share of the preparation (the rope'd
-// columns) and compute the next chunk's rotation angles while the others run the
-// matrix work.  A chunk is two phases with a barrier after each:
+// The contractions over d_state and over the keys run on bf16 matrix cores with every
+// float32 operand as the exact sum of three bf16 parts and six part products
+// (m3_chunk_common.h): 3/8 of the float32 MFMA's time, and against float64 the same
+// error (8e-8 in the 2-norm, measured at d_state 64 and 128).  The intra-chunk M V keeps
+// v_mfma_f32_16x16x4_f32: its operands are in registers and used once, so splitting them
+// would cost more than it saves.  With float32 MFMA throughout a chunk's matrix phase
+// was bound by them (5.6 of 12.8 k cycles on the busiest SIMD) and the scan took 664 us
+// at B=8, L=4096, H=32, d_state 128; with the parts 517 us (same box).
+//
+// One workgroup of 12 waves per (batch, head) walks the chunks in order.  Output waves
+// 0-2 each own one (query block, key block) item of Y_diag (an S^T block, the causal
+// mask or the decay, M V over its keys).  State waves 4-7 each own 16 columns of the
+// value dimension (a p-tile): h^T[:, p-tile] (all N rows) as 16x16 accumulators, that
+// p-tile's Y_off = Q_r h^T and its state update.  Output and auxiliary waves (8-11) take
+// the preparation's Q/K columns (the rope'd ones and the angles on both), the state
+// waves the gate.  A chunk is two phases with a barrier after each:
 //   preparation  lane = token: biases, rope and key scale into the Q/K tiles; the gate
 //                and store of the previous chunk's Y; the direct-to-LDS loads of the
 //                next chunk's Q and K
@@ -49,22 +54,24 @@ __device__ __forceinline__ void half_incl_scan2(float v[2]) {
 template <typename T, int CS_, int N_, int P_, int R_, int NW_>
 struct Geo : GeoBase<T, CS_, N_, P_, R_, NW_> {
   typedef GeoBase<T, CS_, N_, P_, R_, NW_> B;
-  static constexpr int LDY = B::P + (B::BF ? 8 : 2);       // sY rows (io precision)
+  static constexpr int LDY = B::P;                         // sY rows (swizzled, yoff)
+  // Element (row, col) of a Y tile: the 16-column blocks are exchanged by row / 4, so
+  // that an accumulator tile's stores (rows 4 g + r of lane groups g) miss each other's banks.
+  __device__ static int yoff(int row, int col) { return row * LDY + (col ^ (16 * ((row >> 2) & (B::PT - 1)))); }
   // LDS bytes besides the Q/K staging.  The Q/K staging is double-buffered where it
   // fits; otherwise (rotation width N/2 at d_state 128) it is single-buffered and its
   // loads wait until the preparation phase has consumed it.
-  static constexpr int FIXED = 2 * B::CS * B::LDQ * B::TS + 2 * B::CS * LDY * B::TS + 16 * LDY * B::TS +
+  static constexpr int FIXED = 2 * 3 * B::CS * B::N * 2 + 2 * B::CS * LDY * B::TS + 16 * LDY * B::TS +
                                (2 * B::CS * B::SV + 2 * B::CS * B::SA) * 16 + 2 * 3 * (B::CS + 4) * 4 + 8 * B::N +
-                               2 * 6 * B::CS * 4 + 64;
-  static constexpr bool DBQK = FIXED + 4 * B::CS * B::SQ * 16 <= 160 * 1024 - 512;
+                               2 * 6 * B::CS * 4 + 16 + 4 * B::N;
+  static constexpr bool DBQK = FIXED + 4 * B::CS * B::SQ * 16 <= 160 * 1024;
   static constexpr int NQK = DBQK ? 2 : 1;
   static_assert(B::SPT >= 1 && B::NST % B::PT == 0 && B::LB16 % B::SPT == 0, "state-wave split");
   // Q/K 8-column group k (< QGW) of a wave, or QG for none.  The first groups are the
   // rope columns, and their owner also computes their angles for the next chunk.  Full
-  // pass: the output and auxiliary waves take the first groups, one each, so the angle
-  // work stays off the state waves (the matrix phase ends with them); then the state
-  // waves (which also run the gate in the preparation) and the auxiliary waves take
-  // one each of the rest.  State-only pass
+  // pass: the output and auxiliary waves take the groups, two each, so the angle work
+  // stays off the state waves (the matrix phase ends with them, and they run the gate in
+  // the preparation).  State-only pass
   // (no Q and no Y, so the output waves have no matrix work): the output waves and then
   // the auxiliary waves take the first groups, one each, and the state waves two each
   // of the rest, which halves the angle work per wave.
@@ -77,8 +84,8 @@ struct Geo : GeoBase<T, CS_, N_, P_, R_, NW_> {
       else if (wave >= NWY + NST) g = k == 0 ? NWY + (wave - NWY - NST) : QG;
       else g = NWY + NAUX + 2 * (wave - NWY) + k;
     } else {
-      if (wave < NWY) g = k == 0 ? wave : QG;
-      else if (wave < NWY + NST) g = k == 0 ? NWY + NAUX + (wave - NWY) : QG;
+      if (wave < NWY) g = k == 0 ? wave : NWY + NAUX + wave;
+      else if (wave < NWY + NST) g = QG;
       else g = k == 0 ? NWY + (wave - NWY - NST) : 2 * NWY + NAUX + (wave - NWY - NST);
     }
     return g < QG ? g : QG;
@@ -88,8 +95,8 @@ struct Geo : GeoBase<T, CS_, N_, P_, R_, NW_> {
 template <typename G>
 struct __attribute__((aligned(16))) Smem {
   typedef typename std::conditional<G::BF, bf16, float>::type T;
-  T q[G::CS * G::LDQ];                   // rope'd Q rows
-  T k[G::CS * G::LDQ];                   // rope'd, trapezoid-scaled K rows
+  PlaneTile<G::CS, G::N, true> q;        // rope'd Q rows, in bf16 parts
+  PlaneTile<G::CS, G::N, false> k;       // rope'd, trapezoid-scaled K rows, in bf16 parts
   // Y before the gate, in two parts written by plain stores: the intra-chunk part
   // (output waves, by query block) and Q h^T (state waves, by p-tile; the gate applies
   // its e^{A_cum} row scale)
@@ -176,7 +183,7 @@ void scan_chunked_f32_kernel(ScanArgs a) {
   };
   auto gate = [&](int c) {                 // Y of chunk c -> out
     if (eact && c * CS + erow < L) {
-      const int off = erow * G::LDY + 8 * egrp;
+      const int off = G::yoff(erow, 8 * egrp);
       Vec8<T> ya, yb;
       ya.load(&sm.yd[off]);
       yb.load(&sm.yo[off]);
@@ -189,7 +196,7 @@ void scan_chunked_f32_kernel(ScanArgs a) {
       if (erow >= 16) {                    // rows 16..31: the off-diagonal phase-3 item
         Vec8<T> yc;
         float oc[8];
-        yc.load(&sm.ydo[(erow - 16) * G::LDY + 8 * egrp]);
+        yc.load(&sm.ydo[G::yoff(erow - 16, 8 * egrp)]);
         yc.to_f(oc);
 #pragma unroll
         for (int q = 0; q < 8; ++q) o[q] += oc[q];
@@ -242,7 +249,8 @@ void scan_chunked_f32_kernel(ScanArgs a) {
   constexpr int kScalarWave = SO ? G::NWY + G::NST : G::NW - 1;
   float p_cs[G::QGW][2], p_sn[G::QGW][2];
   float logdec = 0.0f;                     // state-only pass: sum of the chunks' log-decays
-  auto pre = [&](int cc) {
+  auto pre = [&](int cc, auto rope_c) {
+    constexpr bool RP = decltype(rope_c)::value;   // false: none of the caller's groups are rope columns
     const int t0 = cc * CS;
     const int pb = cc & 1;
     const bool tok = lane < CS && t0 + lane < L;
@@ -266,7 +274,7 @@ void scan_chunked_f32_kernel(ScanArgs a) {
 #pragma unroll
     for (int k = 0; k < G::QGW; ++k) {
       const int g = G::template qgroup<SO>(wave, k);
-      if (g < G::QG && 4 * g < R) {
+      if (RP && g < G::QG && 4 * g < R) {
         // two lanes per token (tkn, hf): this lane's pairs 4 g + 2 hf + {0, 1}
         const bool ttok = t0 + tkn < L;
         const float h_dt = ttok ? sm.rs[pb][1][tkn] : 0.0f;
@@ -305,21 +313,18 @@ void scan_chunked_f32_kernel(ScanArgs a) {
   if (nc > 1) stage_ars(1);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  pre(0);
+  pre(0, std::true_type{});
   __syncthreads();   // chunk 0's per-token constants (one wave writes them) before its preparation
 
-  for (int c = 0; c < nc; ++c) {
+  // ---- preparation: the wave's Q/K column groups, two lanes per token: biases, rope,
+  // key scale.  Rows past the sequence end hold stale (finite) inputs: their key scale
+  // is 0, so they add nothing to S or h, and their outputs are never stored.
+  auto prep_groups = [&](int c, auto rope_c) {
+    constexpr bool RP = decltype(rope_c)::value;
     const int t0 = c * CS;
-    const int pc = c & 1;
     const uint4* sq = sm.rq[c % G::NQK];
     const uint4* sk = sm.rk[c % G::NQK];
-    const uint4* sv = sm.rv[pc];
-
-    // ================= preparation =================
-    // Rows past the sequence end hold stale (finite) inputs: their key scale is 0,
-    // so they add nothing to S or h, and their outputs are never stored.
-    // Q/K column groups, two lanes per token: biases, rope, key scale
-    const float hscl = sm.scl[pc][tkn];
+    const float hscl = sm.scl[c & 1][tkn];
 #pragma unroll
     for (int k = 0; k < G::QGW; ++k) {
       const int g = G::template qgroup<SO>(wave, k);
@@ -332,7 +337,7 @@ void scan_chunked_f32_kernel(ScanArgs a) {
                        __uint_as_float(qr.w) + qb.w};
         float kf[4] = {__uint_as_float(kr.x) + kb.x, __uint_as_float(kr.y) + kb.y, __uint_as_float(kr.z) + kb.z,
                        __uint_as_float(kr.w) + kb.w};
-        if (4 * g < R) {
+        if (RP && 4 * g < R) {
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             const float cs = p_cs[k][j], sn = p_sn[k][j];
@@ -347,189 +352,235 @@ void scan_chunked_f32_kernel(ScanArgs a) {
         if (t0 + tkn == L - 1) store4(&sm.fink[col], kf);   // the final carry's key, written after the loop
 #pragma unroll
         for (int e = 0; e < 4; ++e) kf[e] *= hscl;
-        if constexpr (!SO) store4(&sm.q[tkn * G::LDQ + col], qf);
-        store4(&sm.k[tkn * G::LDQ + col], kf);
+        if constexpr (!SO) sm.q.put4(tkn, 2 * g + hf, qf);
+        sm.k.put4(tkn, 2 * g + hf, kf);
       }
     }
-    // gate of the previous chunk (its Y tiles were written before the last barrier),
-    // then Z for this chunk's gate, then the loads of the next chunks: the gate's wait
-    // for Z comes before any of them is in flight
-    if (!SO && c > 0) gate(c - 1);
-    if (!SO) load_z(c);
-    if (G::DBQK && c + 1 < nc) stage_qk(c + 1);
-    __syncthreads();
+  };
 
-    // single-buffered Q/K staging: every wave has read this chunk's rows
-    if (!G::DBQK && c + 1 < nc) stage_qk(c + 1);
-    if (c + 1 < nc) stage_v(c + 1);
-    if (c + 2 < nc) stage_ars(c + 2);
-
-    // ---- phase 3 as (query block lb, key block sb <= lb) items, one per output wave:
-    // three at 32-token chunks, on three SIMDs (each also holds a state wave).  An item
-    // is the 16 x 16 block S^T of keys 16 sb.. against queries 16 lb.., masked -- decayed
-    // off the diagonal block; on it causal, with D + gamma QK on the diagonal -- then
-    // M V over those 16 keys for every p-tile.  The diagonal items write their rows of
-    // Y_diag to yd, the off-diagonal one to ydo, which the gate adds.  The S^T operands
-    // are read four k-steps at a time: in step s of a 16-wide block of the d_state axis,
-    // k slot i/16 of lane i stands for column k0 + 4 (i/16) + s in both operands (the
-    // dot product is the same sum in another order), one 16-byte read per operand per
-    // four MFMAs.
-    auto diag_item = [&](auto lb_c, auto sb_c) {
-      constexpr int lb = decltype(lb_c)::value, sb = decltype(sb_c)::value;
-      static_assert(sb <= lb, "causal items only");
-      // lane-derived addresses are recomputed here, not kept live across the loop
-      int ln = lane;
-      asm volatile("" : "+v"(ln));
-      const int g4l = 4 * (ln >> 4);
-      const int l = 16 * lb + (ln & 15);
-      const float al = sm.ac2[pc][l];
-      const float* kr = &sm.k[(16 * sb + (ln & 15)) * G::LDQ + 4 * (ln >> 4)];
-      const float* qr = &sm.q[(16 * lb + (ln & 15)) * G::LDQ + 4 * (ln >> 4)];
-      f32x4 st = {0.0f, 0.0f, 0.0f, 0.0f};
+  // ---- phase 3 as (query block lb, key block sb <= lb) items, one per output wave:
+  // three at 32-token chunks, on three SIMDs (each also holds a state wave).  An item
+  // is the 16 x 16 block S^T of keys 16 sb.. against queries 16 lb.., masked -- decayed
+  // off the diagonal block; on it causal, with D + gamma QK on the diagonal -- then
+  // M V over those 16 keys for every p-tile.  The diagonal items write their rows of
+  // Y_diag to yd, the off-diagonal one to ydo, which the gate adds.  The S^T operands
+  // are read four k-steps at a time: in step s of a 16-wide block of the d_state axis,
+  // k slot i/16 of lane i stands for column k0 + 4 (i/16) + s in both operands (the
+  // dot product is the same sum in another order), one 16-byte read per operand per
+  // four MFMAs.
+  auto diag_item = [&](auto lb_c, auto sb_c, int c) {
+    const int pc = c & 1;
+    const uint4* sv = sm.rv[pc];
+    constexpr int lb = decltype(lb_c)::value, sb = decltype(sb_c)::value;
+    static_assert(sb <= lb, "causal items only");
+    // lane-derived addresses are recomputed here, not kept live across the loop
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int g4l = 4 * (ln >> 4);
+    const int l = 16 * lb + (ln & 15);
+    const float al = sm.ac2[pc][l];
+    f32x4 st = {0.0f, 0.0f, 0.0f, 0.0f}, stl = {0.0f, 0.0f, 0.0f, 0.0f};
+    Parts8 ka[1] = {sm.k.row(16 * sb, 0, ln)}, qa[1] = {sm.q.row(16 * lb, 0, ln)};
 #pragma unroll
-      for (int k0 = 0; k0 < N; k0 += 16) {
-        const float4 ka = *reinterpret_cast<const float4*>(kr + k0);
-        const float4 qa = *reinterpret_cast<const float4*>(qr + k0);
-        st = W::mma(ka.x, qa.x, st);
-        st = W::mma(ka.y, qa.y, st);
-        st = W::mma(ka.z, qa.z, st);
-        st = W::mma(ka.w, qa.w, st);
+    for (int q = 0; q < N / 32; ++q) {
+      Parts8 kn[1], qn[1];
+      if (q + 1 < N / 32) {
+        kn[0] = sm.k.row(16 * sb, q + 1, ln);
+        qn[0] = sm.q.row(16 * lb, q + 1, ln);
       }
-      const int s0 = 16 * sb + g4l;
-      if constexpr (sb < lb) {
-        // off-diagonal block: e^{A_l - A_s} = e^{A_l - A_e} e^{A_e - A_s}, both <= 1
-        const float f = exp2_fast(fminf(al - sm.ac2[pc][16 * sb + 15], 0.0f));
-        const float4 gg = *reinterpret_cast<const float4*>(&sm.g16[pc][s0]);
-        st[0] *= f * gg.x; st[1] *= f * gg.y; st[2] *= f * gg.z; st[3] *= f * gg.w;
-      } else {
-        // diagonal block: causal decay below the diagonal; on it, D plus the
-        // QK skip gamma_l (q_l . k_l) (the stored key carries the scale)
-        const float dgl = sm.dg[pc][l];
-        const float4 as = *reinterpret_cast<const float4*>(&sm.ac2[pc][s0]);
-        const float asv[4] = {as.x, as.y, as.z, as.w};
+      __builtin_amdgcn_sched_barrier(0);
+      mma_parts<1>(ka, qa, &st, &stl);
+      if (q + 1 < N / 32) {
+        ka[0] = kn[0];
+        qa[0] = qn[0];
+      }
+    }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float v = st[r] * exp2_fast(fminf(al - asv[r], 0.0f));
-          st[r] = (s0 + r < l) ? v : (s0 + r == l ? Dh + st[r] * dgl : 0.0f);
-        }
+    for (int r = 0; r < 4; ++r) st[r] += stl[r];
+    const int s0 = 16 * sb + g4l;
+    if constexpr (sb < lb) {
+      // off-diagonal block: e^{A_l - A_s} = e^{A_l - A_e} e^{A_e - A_s}, both <= 1
+      const float f = exp2_fast(fminf(al - sm.ac2[pc][16 * sb + 15], 0.0f));
+      const float4 gg = *reinterpret_cast<const float4*>(&sm.g16[pc][s0]);
+      st[0] *= f * gg.x; st[1] *= f * gg.y; st[2] *= f * gg.z; st[3] *= f * gg.w;
+    } else {
+      // diagonal block: causal decay below the diagonal; on it, D plus the
+      // QK skip gamma_l (q_l . k_l) (the stored key carries the scale)
+      const float dgl = sm.dg[pc][l];
+      const float4 as = *reinterpret_cast<const float4*>(&sm.ac2[pc][s0]);
+      const float asv[4] = {as.x, as.y, as.z, as.w};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = st[r] * exp2_fast(fminf(al - asv[r], 0.0f));
+        st[r] = (s0 + r < l) ? v : (s0 + r == l ? Dh + st[r] * dgl : 0.0f);
       }
-      // M V: the A operand is the masked block itself (lane i, reg j: query l, key
-      // 16 sb + 4 (i/16) + j), matched by V's rows
-      f32x4 yd[G::PT];
+    }
+    // M V: the A operand is the masked block itself (lane i, reg j: query l, key
+    // 16 sb + 4 (i/16) + j), matched by V's rows
+    f32x4 yd[G::PT];
+#pragma unroll
+    for (int pt = 0; pt < G::PT; ++pt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) yd[pt][r] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int pt = 0; pt < G::PT; ++pt)
+        yd[pt] = W::mma(st[j], W::template vdiag<G::SV>(sv, 16 * pt, 16 * sb, j, ln), yd[pt]);
+    T* dst = sb == lb ? sm.yd + 16 * lb * G::LDY : sm.ydo;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) yd[pt][r] = 0.0f;
+    for (int pt = 0; pt < G::PT; ++pt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int pt = 0; pt < G::PT; ++pt)
-          yd[pt] = W::mma(st[j], W::template vdiag<G::SV>(sv, 16 * pt, 16 * sb, j, ln), yd[pt]);
-      T* dst = sb == lb ? sm.yd + 16 * lb * G::LDY : sm.ydo;
-#pragma unroll
-      for (int pt = 0; pt < G::PT; ++pt)
-#pragma unroll
-        for (int r = 0; r < 4; r += 2)
-          store_pair(&dst[(g4l + r) * G::LDY + 16 * pt + (ln & 15)],
-                     &dst[(g4l + r + 1) * G::LDY + 16 * pt + (ln & 15)], yd[pt][r], yd[pt][r + 1]);
+      for (int r = 0; r < 4; r += 2)
+        store_pair(&dst[G::yoff(g4l + r, 16 * pt + (ln & 15))], &dst[G::yoff(g4l + r + 1, 16 * pt + (ln & 15))],
+                   yd[pt][r], yd[pt][r + 1]);
+  };
+  auto state_work = [&](int c) {
+    const int pc = c & 1;
+    const uint4* sv = sm.rv[pc];
+    // lane-derived addresses are recomputed here, not kept live across the loop
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int g4l = 4 * (ln >> 4), pc_l = 16 * pr + (ln & 15);
+    // the state update's decay and per-token weights are read before this wave's
+    // stores (a read issued after them would wait for them too)
+    const float dec = sm.dec[pc];
+    float wv[8];                         // of tokens 8 (lane/16) + 0..7
+    auto load_wv = [&]() {
+      const float* w = &sm.wdec[pc][8 * (ln >> 4)];
+      const float4 w0 = *reinterpret_cast<const float4*>(w), w1 = *reinterpret_cast<const float4*>(w + 4);
+      wv[0] = w0.x; wv[1] = w0.y; wv[2] = w0.z; wv[3] = w0.w;
+      wv[4] = w1.x; wv[5] = w1.y; wv[6] = w1.z; wv[7] = w1.w;
     };
-    if (!SO && ywave) {                 // the state-only pass has no Y_diag
-      static_assert(G::LB16 == 2 && G::NWY >= 3, "three phase-3 items on three output waves");
-      if (wave == 0) diag_item(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-      if (wave == 1) diag_item(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
-      if (wave == 2) diag_item(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{});
-    } else if (swave) {
-      // the state update's decay and per-token weights are read before this wave's
-      // stores (a read issued after them would wait for them too)
-      const float dec = sm.dec[pc];
-      float wv[CS / W::KSTEP][W::WN];
-      auto load_wv = [&]() {
+    // ---- phase 6: Y_off = Q_r h^T for my p-tile, query blocks lb = part (mod SPT)
+    if constexpr (!SO) {
+    constexpr int NLB = G::LB16 / G::SPT;
+    f32x4 yo[NLB], yl[NLB];
 #pragma unroll
-        for (int ks = 0; ks < CS / W::KSTEP; ++ks) W::load_w(&sm.wdec[pc][W::ktok(ks * W::KSTEP, lane)], wv[ks]);
-      };
-      // ---- phase 6: Y_off = Q_r h^T for my p-tile, query blocks lb = part (mod SPT)
-      if constexpr (!SO) {
-      typename W::frag hf[G::BF ? N / 32 : 1];
-      if constexpr (G::BF) {
+    for (int i = 0; i < NLB; ++i)
 #pragma unroll
-        for (int q = 0; q < N / 32; ++q) hf[q] = W::hfrag(hs[2 * q], hs[2 * q + 1]);
-      }
-      constexpr int NLB = G::LB16 / G::SPT;
-      f32x4 yo[NLB];
+      for (int r = 0; r < 4; ++r) yo[i][r] = yl[i][r] = 0.0f;
+    // a step's query operands are requested before the state's split, which hides them
 #pragma unroll
-      for (int i = 0; i < NLB; ++i)
+    for (int q = 0; q < N / 32; ++q) {
+      Parts8 qa[NLB], hp[NLB];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) yo[i][r] = 0.0f;
-      if constexpr (G::BF) {
-        // per k-step the query blocks' fragments, then their chains side by side
+      for (int i = 0; i < NLB; ++i) qa[i] = sm.q.row(16 * (part + G::SPT * i), q, ln);
+      __builtin_amdgcn_sched_barrier(0);
+      const float hv[8] = {hs[2 * q][0], hs[2 * q][1], hs[2 * q][2], hs[2 * q][3],
+                           hs[2 * q + 1][0], hs[2 * q + 1][1], hs[2 * q + 1][2], hs[2 * q + 1][3]};
+      hp[0] = split8(hv);
 #pragma unroll
-        for (int q = 0; q < N / 32; ++q) {
-          typename W::frag qa[NLB];
+      for (int i = 1; i < NLB; ++i) hp[i] = hp[0];
+      mma_parts<NLB>(qa, hp, yo, yl);
+    }
+    load_wv();
 #pragma unroll
-          for (int i = 0; i < NLB; ++i) qa[i] = W::qoff(sm.q, G::LDQ, 16 * (part + G::SPT * i), 32 * q, lane);
+    for (int i = 0; i < NLB; ++i) {
+      const int lb = part + G::SPT * i;
 #pragma unroll
-          for (int i = 0; i < NLB; ++i) yo[i] = W::mma(qa[i], hf[q], yo[i]);
-        }
-      } else {
-#pragma unroll
-        for (int nb = 0; nb < G::NB16; ++nb)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int i = 0; i < NLB; ++i) {
-              const int l = 16 * (part + G::SPT * i) + (lane & 15);
-              yo[i] = W::mma(sm.q[l * G::LDQ + 16 * nb + g4 + r], hs[nb][r], yo[i]);
-            }
-      }
+      for (int r = 0; r < 4; r += 2)
+        store_pair(&sm.yo[G::yoff(16 * lb + g4l + r, pc_l)], &sm.yo[G::yoff(16 * lb + g4l + r + 1, pc_l)],
+                   yo[i][r] + yl[i][r], yo[i][r + 1] + yl[i][r + 1]);
+    }
+    } else {
       load_wv();
+    }
+    // ---- phases 4-5: h <- e^{A_end} h + K_s^T (w V) for my p-tile
+    // the state entering chunk c, [p][n], for the backward
+    if constexpr (SO || SAVE) {
+      if (a.chunk_h && part == 0) {
+        T* dst = reinterpret_cast<T*>(a.chunk_h) + (ch0 + c) * P * N;
 #pragma unroll
-      for (int i = 0; i < NLB; ++i) {
-        const int lb = part + G::SPT * i;
-#pragma unroll
-        for (int r = 0; r < 4; r += 2)
-          store_pair(&sm.yo[(16 * lb + g4 + r) * G::LDY + pcol], &sm.yo[(16 * lb + g4 + r + 1) * G::LDY + pcol],
-                     yo[i][r], yo[i][r + 1]);
-      }
-      } else {
-        load_wv();
-      }
-      // ---- phases 4-5: h <- e^{A_end} h + K_s^T (w V) for my p-tile
-      // the state entering chunk c, [p][n], for the backward
-      if constexpr (SO || SAVE) {
-        if (a.chunk_h && part == 0) {
-          T* dst = reinterpret_cast<T*>(a.chunk_h) + (ch0 + c) * P * N;
-#pragma unroll
-          for (int nb = 0; nb < G::NB16; ++nb) {
-            const float hv[4] = {hs[nb][0], hs[nb][1], hs[nb][2], hs[nb][3]};
-            store4(dst + saved_tile_off<N>(pr, nb, lane), hv);
-          }
+        for (int nb = 0; nb < G::NB16; ++nb) {
+          const float hv[4] = {hs[nb][0], hs[nb][1], hs[nb][2], hs[nb][3]};
+          store4(dst + saved_tile_off<N>(pr, nb, ln), hv);
         }
-      }
-#pragma unroll
-      for (int nb = 0; nb < G::NB16; ++nb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) hs[nb][r] *= dec;
-#pragma unroll
-      for (int ks = 0; ks < CS / W::KSTEP; ++ks) {
-        const typename W::frag vb = W::scale(W::template vstate<G::SV>(sv, 16 * pr, ks * W::KSTEP, lane), wv[ks]);
-#pragma unroll
-        for (int nb = 0; nb < G::NB16; ++nb)
-          hs[nb] = W::mma(W::kstate(sm.k, G::LDQ, ks * W::KSTEP, 16 * nb, lane), vb, hs[nb]);
       }
     }
-    if (c + 1 < nc) pre(c + 1);
-    __builtin_amdgcn_s_waitcnt(0);   // this wave's staged loads and gate stores are done
-    __syncthreads();
-  }
-  if (!SO && nc > 0) gate(nc - 1);
-
-  final_kv<G>(a, sm, cb, tid);
-  if (a.fin_h && fin_here && swave && part == 0) {
 #pragma unroll
     for (int nb = 0; nb < G::NB16; ++nb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) a.fin_h[((long)ci_out * P + pcol) * N + 16 * nb + g4 + r] = hs[nb][r];
+      for (int r = 0; r < 4; ++r) hs[nb][r] *= dec;
+    // the key operands, two state tiles at a time, requested a step ahead
+    Parts8 kp[2] = {sm.k.col(0, 0, ln), sm.k.col(0, 1, ln)};
+    float wx[8];                         // w V: tokens 8 (lane/16) + 0..7, column pcol
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      wx[j] = *staged_elem<G::SV, float>(sv, 8 * (ln >> 4) + j, 16 * pr + (ln & 15)) * wv[j];
+    Parts8 wp[2];
+    wp[0] = wp[1] = split8(wx);
+#pragma unroll
+    for (int nb = 0; nb < G::NB16; nb += 2) {
+      Parts8 kn[2];
+      if (nb + 2 < G::NB16) {
+        kn[0] = sm.k.col(0, nb + 2, ln);
+        kn[1] = sm.k.col(0, nb + 3, ln);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      mma_parts<2>(kp, wp, &hs[nb], &hs[nb]);
+      if (nb + 2 < G::NB16) {
+        kp[0] = kn[0];
+        kp[1] = kn[1];
+      }
+    }
+  };
+
+  // ---- the chunk loop, one per role: the roles share no loop-carried registers (the
+  // state accumulators live only in the state waves' loop), and every loop passes the
+  // same two barriers per chunk.  At rope widths up to 8 NWY the state waves own no
+  // rope group (they take groups from NWY + NAUX on).
+  const std::integral_constant<bool, SO && (R > 4 * (G::NWY + G::NAUX))> rst{};
+  if (ywave) {
+    for (int c = 0; c < nc; ++c) {
+      prep_groups(c, std::true_type{});
+      if (G::DBQK && c + 1 < nc) stage_qk(c + 1);
+      __syncthreads();
+      if (c + 1 < nc) stage_v(c + 1);
+      if (c + 2 < nc) stage_ars(c + 2);
+      if constexpr (!SO) {              // the state-only pass has no Y_diag
+        static_assert(G::LB16 == 2 && G::NWY >= 3, "three phase-3 items on three output waves");
+        if (wave == 0) diag_item(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, c);
+        if (wave == 1) diag_item(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, c);
+        if (wave == 2) diag_item(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{}, c);
+      }
+      if (c + 1 < nc) pre(c + 1, std::true_type{});
+      __builtin_amdgcn_s_waitcnt(0);   // this wave's staged loads are done
+      __syncthreads();
+    }
+  } else if (swave) {
+    for (int c = 0; c < nc; ++c) {
+      prep_groups(c, rst);
+      // gate of the previous chunk (its Y tiles were written before the last barrier),
+      // then Z for this chunk's gate
+      if (!SO && c > 0) gate(c - 1);
+      if (!SO) load_z(c);
+      __syncthreads();
+      state_work(c);
+      if (c + 1 < nc) pre(c + 1, rst);
+      __builtin_amdgcn_s_waitcnt(0);   // this wave's Z and gate stores are done
+      __syncthreads();
+    }
+    if (!SO && nc > 0) gate(nc - 1);
+    if (a.fin_h && fin_here && part == 0) {
+#pragma unroll
+      for (int nb = 0; nb < G::NB16; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a.fin_h[((long)ci_out * P + pcol) * N + 16 * nb + g4 + r] = hs[nb][r];
+    }
+  } else {
+    for (int c = 0; c < nc; ++c) {
+      prep_groups(c, std::true_type{});
+      __syncthreads();
+      // single-buffered Q/K staging: every wave has read this chunk's rows
+      if (!G::DBQK && c + 1 < nc) stage_qk(c + 1);
+      if (c + 1 < nc) pre(c + 1, std::true_type{});
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+    }
   }
+
+  final_kv<G>(a, sm, cb, tid);
   if constexpr (SO) {
     if (a.fin_logdec && fin_here && wave == kScalarWave && lane == 0) a.fin_logdec[ci_out] = logdec;
   }
