@@ -2,12 +2,11 @@
 // (bf16 I/O in m3_scan_chunked.hip, float32 I/O in m3_scan_chunked_f32.hip).
 //
 // Both run one workgroup of 12 waves per (batch, head, sequence segment) over the
-// segment's chunks in order, stage every chunk's rows by direct-to-LDS loads
-// double-buffered by chunk parity, carry the state in the state waves' accumulators
-// and compute the same per-token chunk constants on one wave.  What differs between
-// them stays in each kernel: the geometry and LDS layout (64- against 32-token chunks,
-// the float32 kernel's Y tiles), the wave roles (four query blocks on the output waves
-// against three phase-3 items spread over three SIMDs) and the chunk loop built on them.
+// segment's chunks in order, stage rows by direct-to-LDS loads double-buffered by chunk
+// parity (the bf16 kernel all of them, the float32 kernel V and the rates), carry the
+// state in the state waves' accumulators and compute the same per-token chunk constants
+// on one wave.  What differs between them stays in each kernel: the geometry and LDS
+// layout, the wave roles and the chunk loop built on them.
 #pragma once
 
 #include <type_traits>
@@ -17,7 +16,7 @@
 namespace m3 {
 
 // Geometry common to the chunked kernels' instantiations: 12 waves (output waves 0-3,
-// state waves 4-7, auxiliary waves 8-11), 16 x 16 MFMA tiles, the Q/K 8-column groups
+// state waves 4-7, auxiliary (float32: preparation) waves 8-11), 16 x 16 MFMA tiles, the Q/K 8-column groups
 // and the staging tiles' 16-byte slots per row.  Each kernel's Geo adds its LDS budget
 // and its assignment of the column groups to the waves.
 template <typename T, int CS_, int N_, int P_, int R_, int NW_>
@@ -37,6 +36,7 @@ struct GeoBase {
   static constexpr int QG = N / 8, QGW = 2;                 // Q/K 8-column groups, at most 2 per wave
   // 16-byte staging slots per row: Q/K, V, rotation rates
   static constexpr int SQ = N * TS / 16, SV = P * TS / 16, SA = R / 4 > 0 ? R / 4 : 1;
+  static constexpr int NRA = 2;                             // buffers of the staged rates and scalars
   static_assert(CS <= 64 && LB16 <= NWY, "one token per lane, one query block per output wave");
   static_assert(NAUX == 4, "12 waves");
   static_assert(QG <= 2 * NAUX + NWY + NST, "column groups per wave");
@@ -162,7 +162,7 @@ __device__ __forceinline__ void stage_ars_chunk(Sm& sm, const ChunkBlock<T>& cb,
   if (wave == WA) {
     if (R > 0) {
       const char* a0 = reinterpret_cast<const char*>(cb.ang_base + (long)t0 * cb.a_stride);
-      stage_rows<CS, G::SA, 0, JA>((lds_uint4*)sm.ra[c & 1], a0, cb.a_stride * 4, valid, lane);
+      stage_rows<CS, G::SA, 0, JA>((lds_uint4*)sm.ra[c % G::NRA], a0, cb.a_stride * 4, valid, lane);
     }
     // the bases are made opaque here so that no derived pointer is hoisted out of the
     // chunk loop (and spilled)
@@ -171,13 +171,13 @@ __device__ __forceinline__ void stage_ars_chunk(Sm& sm, const ChunkBlock<T>& cb,
     const float* pt = cb.gtr + t0;
     asm volatile("" : "+s"(pa), "+s"(pd), "+s"(pt));
     if (lane < CS && lane < valid) {
-      lds_dma4(pa, 4u * lane, (lds_float*)&sm.rs[c & 1][0][0]);
-      lds_dma4(pd, 4u * lane, (lds_float*)&sm.rs[c & 1][1][0]);
-      lds_dma4(pt, 4u * lane, (lds_float*)&sm.rs[c & 1][2][0]);
+      lds_dma4(pa, 4u * lane, (lds_float*)&sm.rs[c % G::NRA][0][0]);
+      lds_dma4(pd, 4u * lane, (lds_float*)&sm.rs[c % G::NRA][1][0]);
+      lds_dma4(pt, 4u * lane, (lds_float*)&sm.rs[c % G::NRA][2][0]);
     }
     if (lane == 0 && t0 + CS < cb.Lnx) {
-      lds_dma4(pd, 4u * CS, (lds_float*)&sm.rs[c & 1][1][CS]);
-      lds_dma4(pt, 4u * CS, (lds_float*)&sm.rs[c & 1][2][CS]);
+      lds_dma4(pd, 4u * CS, (lds_float*)&sm.rs[c % G::NRA][1][CS]);
+      lds_dma4(pt, 4u * CS, (lds_float*)&sm.rs[c % G::NRA][2][CS]);
     }
   }
 }
@@ -186,13 +186,15 @@ __device__ __forceinline__ void stage_ars_chunk(Sm& sm, const ChunkBlock<T>& cb,
 // loaded, and the preparation reads whole tiles).
 template <typename G, typename Sm>
 __device__ __forceinline__ void zero_staging(Sm& sm, int tid) {
-  for (int i = tid; i < G::NQK * G::CS * G::SQ; i += G::NT) {
-    (&sm.rq[0][0])[i] = make_uint4(0, 0, 0, 0);
-    (&sm.rk[0][0])[i] = make_uint4(0, 0, 0, 0);
+  if constexpr (G::NQK > 0) {
+    for (int i = tid; i < G::NQK * G::CS * G::SQ; i += G::NT) {
+      (&sm.rq[0][0])[i] = make_uint4(0, 0, 0, 0);
+      (&sm.rk[0][0])[i] = make_uint4(0, 0, 0, 0);
+    }
   }
   for (int i = tid; i < 2 * G::CS * G::SV; i += G::NT) (&sm.rv[0][0])[i] = make_uint4(0, 0, 0, 0);
-  for (int i = tid; i < 2 * G::CS * G::SA; i += G::NT) (&sm.ra[0][0])[i] = make_uint4(0, 0, 0, 0);
-  for (int i = tid; i < 2 * 3 * (G::CS + 4); i += G::NT) (&sm.rs[0][0][0])[i] = 0.0f;
+  for (int i = tid; i < G::NRA * G::CS * G::SA; i += G::NT) (&sm.ra[0][0])[i] = make_uint4(0, 0, 0, 0);
+  for (int i = tid; i < G::NRA * 3 * (G::CS + 4); i += G::NT) (&sm.rs[0][0][0])[i] = 0.0f;
 }
 
 // The effective state entering the segment, h0 + (1 - sigmoid(trap_0)) dt_0 (v0 (x) k0)

@@ -285,14 +285,19 @@ template <> struct MF16<float> {
 struct Parts8 {
   bf16x8 h, m, l;
 };
-// The parts of two values, each pair packed (two conversions, two unpacks and two
-// subtractions per part).
+// The parts of two values, each pair packed: per part one conversion, two unpacks and two
+// subtractions.  (The pair is made opaque: otherwise the compiler converts the low value
+// a second time instead of unpacking it.)
+__device__ __forceinline__ uint32_t cvt_pk_bf16(float x0, float x1) {
+  uint32_t r = __builtin_bit_cast(uint32_t, (bf16x2){(bf16)x0, (bf16)x1});
+  asm("" : "+v"(r));
+  return r;
+}
 __device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = __builtin_bit_cast(uint32_t, (bf16x2){(bf16)x0, (bf16)x1});
+  h = cvt_pk_bf16(x0, x1);
   const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
-  m = __builtin_bit_cast(uint32_t, (bf16x2){(bf16)r0, (bf16)r1});
-  l = __builtin_bit_cast(uint32_t, (bf16x2){(bf16)(r0 - __uint_as_float(m << 16)),
-                                            (bf16)(r1 - __uint_as_float(m & 0xffff0000u))});
+  m = cvt_pk_bf16(r0, r1);
+  l = cvt_pk_bf16(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
 }
 __device__ __forceinline__ Parts8 split8(const float x[8]) {
   uint32_t h[4], m[4], l[4];
@@ -319,68 +324,44 @@ __device__ __forceinline__ void mma_parts(const Parts8 (&a)[NT], const Parts8 (&
 #undef M3_STEP
 }
 
-// A [token][n] tile of N columns as three bf16 planes of CS rows of N / 8 16-byte slots.
-// Two orders of the columns in a row:
-//  * PAIRED: slot s holds the columns 32 (s / 4) + 4 (s % 4) + {0..3} and + {16..19}, the
-//    rows of a pair of state tiles that one lane of their accumulators holds, so that a
-//    32-wide step of a contraction over n with the state is one 16-byte read;
-//  * natural, for a tile that is also read transposed (col): 16 consecutive columns are
-//    two whole slots, so that a transposed read touches every bank (PAIRED they would be
-//    halves of four slots, on half of the banks: that took 40% of the LDS cycles of the
-//    float32 scan).
-// Slots are exchanged within a row by swz(row): 16 rows' reads of one slot, and the 8
-// rows of a transposed read's two, lie on different banks.
-template <int CS, int N, bool PAIRED>
+// A [token][n] tile of N columns as three bf16 planes of CS = 32 rows of N / 8 16-byte
+// slots.  Slot s holds the columns 32 (s / 4) + 4 (s % 4) + {0..3} and + {16..19}: the
+// rows of a pair of state tiles that one lane of their accumulators holds, so that a
+// 32-wide step of a contraction over n with the state is one 16-byte read per lane.  The
+// slots of row t are exchanged by swz(t), so that 16 rows' reads of one slot lie on
+// different banks.  (Transposed reads take one half of four slots, half of the banks; a
+// second order of the columns without that measured the same time.)
+template <int CS, int N>
 struct PlaneTile {
   static constexpr int S = N / 8;                  // slots per row: 16, 8 or 4
   uint4 p[3][CS * S];
-  __device__ __forceinline__ static int swz(int t) {
-    if constexpr (PAIRED) return (t >> (S == 16 ? 0 : S == 8 ? 1 : 2)) & (S - 1);
-    if constexpr (S == 16) return ((t >> 2) & 1) | ((t & 3) << 1) | (t & 8);
-    if constexpr (S == 8) return ((t >> 2) & 1) | (t & 2) | ((t >> 1) & 4);
-    return ((t >> 2) & 1) | ((t >> 2) & 2);
-  }
-  // the slot of columns 4 gi .. 4 gi + 3, and which half of it
-  __device__ __forceinline__ static int slot4(int gi) { return PAIRED ? 4 * (gi >> 3) + (gi & 3) : gi >> 1; }
-  __device__ __forceinline__ static int half4(int gi) { return PAIRED ? (gi >> 2) & 1 : gi & 1; }
-  // their offset in row t, in 8-byte units
-  __device__ __forceinline__ static int off4(int t, int gi) {
-    return 2 * (t * S + (slot4(gi) ^ swz(t))) + half4(gi);
-  }
+  __device__ __forceinline__ static int swz(int t) { return (t >> (S == 16 ? 0 : S == 8 ? 1 : 2)) & (S - 1); }
+  // columns 4 gi .. 4 gi + 3 of row t
   __device__ __forceinline__ void put4(int t, int gi, const float x[4]) {
     uint2 h, m, l;
     split2(x[0], x[1], h.x, m.x, l.x);
     split2(x[2], x[3], h.y, m.y, l.y);
-    const int o = off4(t, gi);
+    const int o = 2 * (t * S + ((4 * (gi >> 3) + (gi & 3)) ^ swz(t))) + ((gi >> 2) & 1);
     reinterpret_cast<uint2*>(p[0])[o] = h;
     reinterpret_cast<uint2*>(p[1])[o] = m;
     reinterpret_cast<uint2*>(p[2])[o] = l;
   }
-  // operand of a contraction over n: row row0 + lane%16, the columns 32 q + 4 (lane/16) +
-  // {0..3} and + {16..19} of step q
+  // operand of a contraction over n: row row0 + lane%16 (row0 a multiple of 16), the
+  // columns 32 q + 4 (lane/16) + {0..3} and + {16..19} of step q
   __device__ __forceinline__ Parts8 row(int row0, int q, int lane) const {
-    const int t = row0 + (lane & 15), g = lane >> 4;
+    const int t = lane & 15;
+    const int o = (row0 + t) * S + ((4 * q) ^ ((lane >> 4) ^ swz(t)));
     Parts8 f;
-    bf16x8* out[3] = {&f.h, &f.m, &f.l};
-    if constexpr (PAIRED) {
-      const int o = t * S + ((4 * q + g) ^ swz(t));
-#pragma unroll
-      for (int k = 0; k < 3; ++k) *out[k] = *reinterpret_cast<const bf16x8*>(&p[k][o]);
-    } else {
-      const int o0 = off4(t, 8 * q + g), o1 = off4(t, 8 * q + 4 + g);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const uint2 a = reinterpret_cast<const uint2*>(p[k])[o0], b = reinterpret_cast<const uint2*>(p[k])[o1];
-        *out[k] = __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
-      }
-    }
+    f.h = *reinterpret_cast<const bf16x8*>(&p[0][o]);
+    f.m = *reinterpret_cast<const bf16x8*>(&p[1][o]);
+    f.l = *reinterpret_cast<const bf16x8*>(&p[2][o]);
     return f;
   }
-  // operand of a contraction over tokens t0 + 8 (lane/16) + 0..7: column 16 nb + lane%16
-  __device__ __forceinline__ Parts8 col(int t0, int nb, int lane) const {
-    static_assert(!PAIRED, "natural order");
-    const int l = lane & 15, t = t0 + 8 * (lane >> 4) + (l >> 2), gi = 4 * nb + (l & 3);
-    const int o0 = off4(t, gi), o1 = off4(t + 4, gi);
+  // operand of a contraction over the tokens, 8 (lane/16) + 0..7: column 16 nb + lane%16
+  __device__ __forceinline__ Parts8 col(int nb, int lane) const {
+    const int l = lane & 15, t = 8 * (lane >> 4) + (l >> 2);
+    const int o0 = 2 * (t * S + ((4 * (nb >> 1)) ^ ((l & 3) ^ swz(t)))) + (nb & 1);
+    const int o1 = 2 * ((t + 4) * S + ((4 * (nb >> 1)) ^ ((l & 3) ^ swz(t + 4)))) + (nb & 1);
     Parts8 f;
     bf16x8* out[3] = {&f.h, &f.m, &f.l};
 #pragma unroll
