@@ -96,7 +96,8 @@ int m3_chunk_scan_fwd_carry(const void* Q, const void* K, const void* V,
  * Device workspace (bytes) that m3_chunk_scan_fwd_ws uses to split each sequence
  * into segments running on separate compute units; 0 when the shape runs as one
  * pass.  The split pays off when B*H is well below the compute-unit count
- * (single-sequence prefill, long context).  Hqk does not matter.  No counterpart in the
+ * (single-sequence prefill, long context); with this much room or more the library
+ * chooses the segments, or one pass, by a time model.  Hqk does not matter.  No counterpart in the
  * reference, whose long-context forward passes states in blocks inside its kernel
  * (src/base_model/models/mamba3_pallas.py:679-727).
  */

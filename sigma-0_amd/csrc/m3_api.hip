@@ -9,6 +9,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "../../include/mamba3_layer.h"
@@ -65,7 +66,17 @@ int m3_chunk_scan_impl(int io_dtype, int N, int P, int R, int chunk_size) {
 size_t m3_chunk_scan_ws_bytes(int B, int L, int H, int N, int P, int R, int chunk_size, int io_dtype) {
   if ((io_dtype != M3_DTYPE_F32 && io_dtype != M3_DTYPE_BF16) || B <= 0 || L <= 0 || H <= 0 || chunk_size <= 0)
     return 0;
-  return m3::scan_split_ws_bytes(io_dtype == M3_DTYPE_BF16, B, L, H, N, P, R, chunk_size);
+  const size_t reserved = m3::scan_split_ws_bytes(io_dtype == M3_DTYPE_BF16, B, L, H, N, P, R, chunk_size);
+  if (reserved == 0) return 0;
+  // room for the segments that are chosen with enough of it, the same for both I/O types
+  return std::max({reserved, m3::scan_split_plan_bytes(true, B, L, H, N, P, R, chunk_size),
+                   m3::scan_split_plan_bytes(false, B, L, H, N, P, R, chunk_size)});
+}
+
+size_t m3_scan_split_plan_bytes(int B, int L, int H, int N, int P, int R, int chunk_size, int io_dtype) {
+  if ((io_dtype != M3_DTYPE_F32 && io_dtype != M3_DTYPE_BF16) || B <= 0 || L <= 0 || H <= 0 || chunk_size <= 0)
+    return 0;
+  return m3::scan_split_plan_bytes(io_dtype == M3_DTYPE_BF16, B, L, H, N, P, R, chunk_size);
 }
 
 namespace {
@@ -144,8 +155,11 @@ int scan_fwd(const void* Q, const void* K, const void* V,
       if (ws_bytes < need)
         return fail(M3_E_ARG, "workspace of %zu bytes, the split needs %zu (m3_chunk_scan_ws_bytes)", ws_bytes, need);
       if (!aligned16(ws)) return fail(M3_E_ALIGN, "workspace must be 16-byte aligned");
-      return check_launch(m3::scan_split_launch(a, bf, ws, st), "split chunk scan");
     }
+    // an unaligned workspace where none is promised was never looked at: one pass
+    const int seg_len = ws && aligned16(ws)
+                            ? m3::scan_split_len(bf, B, L, H, N, P, R, chunk_size, ws_bytes) : 0;
+    if (seg_len > 0) return check_launch(m3::scan_split_launch(a, bf, seg_len, ws, st), "split chunk scan");
     return check_launch(m3::scan_chunked_launch(a, bf, st), "chunk scan");
   }
   return check_launch(m3::scan_generic_launch(a, bf, st), "generic scan");

@@ -22,7 +22,7 @@ struct ScanArgs {
   int B, L, H, Hqk, N, P, R, CS;
   // Sequence segments (chunked kernel only): with seg_len > 0 the grid's y index
   // is the segment and block (bh, seg) covers tokens [seg * seg_len,
-  // min(L, (seg + 1) * seg_len)); seg_len is a multiple of 128.  Carries are one per
+  // min(L, (seg + 1) * seg_len)); seg_len is a multiple of 64.  Carries are one per
   // (b, h) (init used by segment 0, fin written by the last segment) or, with
   // init_per_seg / fin_per_seg, one per (b, h, segment) at index bh * nseg + seg.
   int seg_len = 0, init_per_seg = 0, fin_per_seg = 0;
@@ -223,13 +223,21 @@ hipError_t block_norm_bwd_launch(const BlockNormBwdArgs& a, float* dscale, float
 hipError_t nll_launch(float* z, const int* targets, float* loss, long rows, int V, float w, hipStream_t st);
 hipError_t split3_launch(const float* x, void* a, void* b, void* c, long rows, int K, long ld, hipStream_t st);
 
-// Sequence split across compute units: workspace bytes (0 = no split) and launch.
+// Sequence split across compute units.  scan_split_ws_bytes: the least workspace that a
+// split call takes (0: no split is promised).  scan_split_plan_bytes: the one that the
+// fastest segments need (0 = one pass is faster), at least the former where both split.
+// scan_split_len: the segment length for a workspace of ws_bytes (0 = one pass): the
+// fastest, or the reserved one where only that fits.
 size_t scan_split_ws_bytes(bool bf16_io, int B, int L, int H, int N, int P, int R, int CS);
-hipError_t scan_split_launch(const ScanArgs& a, bool bf16_io, void* ws, hipStream_t st);
+size_t scan_split_plan_bytes(bool bf16_io, int B, int L, int H, int N, int P, int R, int CS);
+int scan_split_len(bool bf16_io, int B, int L, int H, int N, int P, int R, int CS, size_t ws_bytes);
+hipError_t scan_split_launch(const ScanArgs& a, bool bf16_io, int seg_len, void* ws, hipStream_t st);
 // The backward's state-only pass (a.chunk_h / a.chunk_th, no initial carry) split the
 // same way: the segments' exit carries, their combine, then every segment's state-only
 // pass from its entering carry writes the states entering its chunks.  Workspace:
-// scan_split_ws_bytes(bf16_io, B, L, H, N, P, R, 64).
+// scan_split_ws_bytes(bf16_io, B, L, H, N, P, R, 64), which is > 0; the segments are those
+// of the forward where they fit in it (one pass included), so that the saved states and
+// the recomputed ones agree bitwise there.
 hipError_t scan_split_state_launch(const ScanArgs& a, bool bf16_io, void* ws, hipStream_t st);
 
 // Arguments of one decode step (layouts in m3_decode.hip).
@@ -256,3 +264,8 @@ bool decode_supported(int N, int P, int R);
 hipError_t decode_step_launch(const DecodeArgs& a, bool in_bf16, bool out_bf16, hipStream_t st);
 
 }  // namespace m3
+
+// Workspace bytes for the split that the library would choose itself (0: none), for the
+// bundled host wrappers, which pass a workspace of this size where the public contract
+// (m3_chunk_scan_ws_bytes) promises a smaller or no split.
+extern "C" size_t m3_scan_split_plan_bytes(int B, int L, int H, int N, int P, int R, int chunk_size, int io_dtype);

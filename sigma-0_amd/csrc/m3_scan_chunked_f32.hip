@@ -675,9 +675,8 @@ bool scan_chunked_f32_supported(int CS_, int N, int P, int R) {
 // shapes whose full pass can also write the chunk states (the backward's float32 shapes)
 #define M3_F32_SAVE_SHAPES(X) X(32, 128, 64, 32) X(32, 128, 64, 64) X(32, 64, 64, 16) X(32, 64, 32, 16)
 
-// the state-only pass of this kernel (the backward's chunk states) at the backward's
-// float32 d_state-128 shapes
-#define M3_F32_STATE_SHAPES(X) X(32, 128, 64, 32) X(32, 128, 64, 64)
+// the state-only pass: the sequence split's first pass and the backward's chunk states
+#define M3_F32_STATE_SHAPES(X) X(32, 128, 64, 32) X(32, 128, 64, 64) X(32, 64, 64, 16) X(32, 64, 32, 16)
 
 bool scan_state_f32_supported(int CS_, int N, int P, int R) {
   const int CS = f32_kernel_chunk(CS_);

@@ -22,6 +22,8 @@
 //
 // This is the reference's sequence-parallel carry algebra (models/mamba3_seqpar.py:
 // 67-110) applied across CUs of one GPU; the extra work is pass 1 (no Q, Y or gate).
+#include <algorithm>
+
 #include "m3_scan.h"
 
 namespace m3 {
@@ -29,25 +31,69 @@ namespace {
 
 constexpr int kCombineThreads = 256;
 constexpr int kTargetBlocks = 256;     // MI355X compute units
-constexpr int kMinSegment = 256;       // tokens
+constexpr int kMinSegment = 64;        // tokens
 constexpr int kMaxRounds = 4;          // rounds of blocks on the chip, at most
 
-// Segment length for a (B, H, L) launch, or 0 for no split.  Segments are whole
-// multiples of 128 tokens, so every interior segment ends on a kernel chunk.
-// Time model: n blocks of len tokens take ceil(n / kTargetBlocks) rounds of len (one
-// block per compute unit), and the state-only pass, which runs every segment but the
-// last, half the full pass's time per token.  The segment count with the least
-// modelled time is taken (the fewest on ties).  For 96 pairs (config 5's layer) that
-// is eight segments, three whole rounds of 256 blocks, rather than two (192 blocks,
-// and 96 in the state-only pass): in the 12-layer stack the layer's three launches
-// took 375 against 417 us.  The model takes a block's time per chunk as fixed; with
-// per-head B/C rows at the same shape, where the chip's memory traffic is larger, the
-// full pass gained less (285 against 293 us) and the three launches took 1.5% longer
-// (0.459 against 0.452 ms by bench.py).
-int seg_len_for(int B, int H, int L) {
+// Modelled time of one pass of n 64-token steps on nb blocks, in ns: rounds of 256 blocks
+// (one per compute unit), each with a start and a time per step that grows a little with
+// the blocks and is at least the time that the chip's memory takes for their bytes
+// (N: d_state; the value dimension counts little).  Slopes and intercepts of passes
+// measured alone (graph replays): per step 2.5 us in bf16 and 6.8 us in float32 at d_state
+// 128 (state-only pass 1.4 and 2.1), 3.4 us in bf16 with every compute unit busy.
+long pass_ns(bool bf16_io, bool state_only, int N, long nb, long n) {
+  const bool wide = N >= 128;
+  const long full[2][2] = {{4100, 6800}, {2020, 2480}};
+  const long so[2][2] = {{1500, 2050}, {950, 1300}};
+  const long base = state_only ? so[bf16_io][wide] : full[bf16_io][wide];
+  const long grow10 = state_only ? 20 : 15;                                  // 0.1 ns per step and block
+  const long mem10 = (state_only ? (wide ? 67 : 43) : (wide ? 133 : 92)) * (bf16_io ? 1 : 2);
+  const long start = state_only ? 5000 : 5700;
+  long t = 0;
+  for (long left = nb; left > 0; left -= kTargetBlocks) {
+    const long b = std::min<long>(left, kTargetBlocks);
+    t += start + n * std::max(base + grow10 * b / 10, mem10 * b / 10);
+  }
+  return t;
+}
+
+// Segment length, or 0 for no split.  Segments are whole multiples of 64 tokens, so every
+// interior segment ends on a kernel chunk (64 tokens in bf16, 32 in float32).  The segment
+// count with the least modelled time (both passes, 10 us for the combine and the gaps, 0.4
+// us per segment) is taken if that is 5% below one pass's.  Measured, in us, one pass / the
+// former rule (reserved_seg_len, which counts no starts) / this one:
+//   bf16  d_state 128: 96 pairs of 1500 tokens 68 / 93 / 68, 128 of 1000 47 / 67 / 47,
+//         24 of 4096 166 / 60 / 60, 32 of 2000 87 / 56 / 46, 24 of 613 40 / 44 / 40
+//   bf16  d_state 64: 16 of 3000 100 / 100 / 34
+//   f32   d_state 128: 24 of 600 66 / 58 / 39;  d_state 64: 16 of 1024 70 / 70 / 31
+int seg_len_for(bool bf16_io, int B, int H, int L, int N) {
   const int bh = B * H;
   if (bh <= 0 || bh * 2 > kTargetBlocks || L < 2 * kMinSegment) return 0;
   const int smax = min(L / kMinSegment, kMaxRounds * kTargetBlocks / bh);
+  const long one = pass_ns(bf16_io, false, N, bh, (L + 63) / 64);
+  int best = 0;
+  long best_cost = one - one / 20;
+  for (int s = 2; s <= smax; ++s) {
+    const int len = ((L + s - 1) / s + 63) / 64 * 64;
+    const long ns = (L + len - 1) / len, n = len / 64;
+    if (ns < 2) continue;
+    const long cost = pass_ns(bf16_io, false, N, bh * ns, n) + pass_ns(bf16_io, true, N, bh * (ns - 1), n) + 10000 +
+                      400 * ns;
+    if (cost < best_cost) {
+      best = len;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+// The segments of the least workspace that a split call takes (scan_split_ws_bytes), which
+// are also those of the backward's state passes: d_state 128 and headdim 64, whole multiples of 128
+// tokens, at least 256; the state-only pass counted as half the full pass's time per
+// token, starts as nothing.
+int reserved_seg_len(int B, int H, int L) {
+  const int bh = B * H;
+  if (bh <= 0 || bh * 2 > kTargetBlocks || L < 512) return 0;
+  const int smax = min(L / 256, kMaxRounds * kTargetBlocks / bh);
   int best = 0;
   long best_cost = 0;
   for (int s = 2; s <= smax; ++s) {
@@ -138,51 +184,69 @@ void seg_combine_kernel(ScanArgs a, int nseg, Carries loc, Carries in) {
     h += (1.0f - 1.0f / (1.0f + expf(-tr0))) * dt0 * a.init_v[(long)bh * P + p] * a.init_k[(long)bh * N + n];
   }
   float th = rope && a.init_theta ? a.init_theta[(long)bh * R + r] : 0.0f;
-  // a segment's values (the element's rope pair of its exit state, its angle advance
-  // and log-decay) are loaded one step ahead of their use, so that the loads overlap
-  // the previous step's arithmetic instead of each step waiting for its own
-  auto load_seg = [&](int i, float2& hp, float& dth, float& ld) {
-    const long ci = c0 + i;
-    hp = *reinterpret_cast<const float2*>(loc.h + ci * P * N + p * N + 2 * r);
-    dth = rope ? loc.th[ci * R + r] : 0.0f;
-    ld = loc.ld[ci];
-  };
-  float2 nhp = make_float2(0.0f, 0.0f);
-  float ndth = 0.0f, nld = 0.0f;
-  if (nseg > 1) load_seg(0, nhp, ndth, nld);
-  for (int i = 0; i + 1 < nseg; ++i) {
-    const float2 hp = nhp;
-    const float dth = ndth, ld = nld;
-    if (i + 2 < nseg) load_seg(i + 1, nhp, ndth, nld);
-    float own = (n & 1) ? hp.y : hp.x;
-    if (rope) {                          // segment-local key frame -> entering frame
-      float sn, cs;
-      sincosf(th, &sn, &cs);
-      own = (n & 1) ? hp.x * sn + hp.y * cs : hp.x * cs - hp.y * sn;
-      const float x = th + dth;
-      th = x - kTwoPi * floorf(x * kInvTwoPi);
+  // the segments' values (the element's rope pair of the exit state, the angle advance
+  // and the log-decay) are loaded kBatch segments at a time before the chain uses them:
+  // the steps are a few operations each, so a load per step would be all latency
+  constexpr int kBatch = 8;
+  for (int i0 = 0; i0 + 1 < nseg; i0 += kBatch) {
+    float2 hp[kBatch];
+    float dth[kBatch], ld[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const long ci = c0 + min(i0 + j, nseg - 2);
+      hp[j] = *reinterpret_cast<const float2*>(loc.h + ci * P * N + p * N + 2 * r);
+      dth[j] = rope ? loc.th[ci * R + r] : 0.0f;
+      ld[j] = loc.ld[ci];
     }
-    h = expf(ld) * h + own;
-    in.h[(c0 + i + 1) * P * N + e] = h;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (i0 + j + 1 >= nseg) break;
+      float own = (n & 1) ? hp[j].y : hp[j].x;
+      if (rope) {                        // segment-local key frame -> entering frame
+        float sn, cs;
+        sincosf(th, &sn, &cs);
+        own = (n & 1) ? hp[j].x * sn + hp[j].y * cs : hp[j].x * cs - hp[j].y * sn;
+        const float x = th + dth[j];
+        th = x - kTwoPi * floorf(x * kInvTwoPi);
+      }
+      h = expf(ld[j]) * h + own;
+      in.h[(c0 + i0 + j + 1) * P * N + e] = h;
+    }
   }
 }
 
 }  // namespace
 
+namespace {
+size_t split_bytes(int len, int B, int L, int H, int N, int P, int R) {
+  return len == 0 ? 0 : carve(nullptr, (long)B * H * ((L + len - 1) / len), N, P, R, nullptr, nullptr);
+}
+bool split_supported(bool bf16_io, int N, int P, int R, int CS) {
+  // shapes without a state-only pass run one pass
+  return scan_state_supported(bf16_io, 64, N, P, R) && scan_chunked_supported(bf16_io, CS, N, P, R);
+}
+}  // namespace
+
 size_t scan_split_ws_bytes(bool bf16_io, int B, int L, int H, int N, int P, int R, int CS) {
-  const int len = seg_len_for(B, H, L);
-  // the model's shapes (d_state 128, headdim 64; bf16, and float32, the I/O the
-  // model's mamba3_siso_triton call hands over) with a state-only pass; others run
-  // one pass
-  if (len == 0 || N != 128 || P != 64 || !scan_state_supported(bf16_io, 64, N, P, R) ||
-      !scan_chunked_supported(bf16_io, CS, N, P, R))
-    return 0;
-  const long bhs = (long)B * H * ((L + len - 1) / len);
-  return carve(nullptr, bhs, N, P, R, nullptr, nullptr);
+  if (N != 128 || P != 64 || !split_supported(bf16_io, N, P, R, CS)) return 0;
+  return split_bytes(reserved_seg_len(B, H, L), B, L, H, N, P, R);
 }
 
-hipError_t scan_split_launch(const ScanArgs& a, bool bf16_io, void* ws, hipStream_t st) {
-  const int len = seg_len_for(a.B, a.H, a.L);
+size_t scan_split_plan_bytes(bool bf16_io, int B, int L, int H, int N, int P, int R, int CS) {
+  if (!split_supported(bf16_io, N, P, R, CS)) return 0;
+  const size_t need = split_bytes(seg_len_for(bf16_io, B, H, L, N), B, L, H, N, P, R);
+  return need == 0 ? 0 : std::max(need, scan_split_ws_bytes(bf16_io, B, L, H, N, P, R, CS));
+}
+
+int scan_split_len(bool bf16_io, int B, int L, int H, int N, int P, int R, int CS, size_t ws_bytes) {
+  if (!split_supported(bf16_io, N, P, R, CS)) return 0;
+  const int len = seg_len_for(bf16_io, B, H, L, N);
+  if (len == 0 || split_bytes(len, B, L, H, N, P, R) <= ws_bytes) return len;
+  const size_t reserved = scan_split_ws_bytes(bf16_io, B, L, H, N, P, R, CS);
+  return reserved > 0 && reserved <= ws_bytes ? reserved_seg_len(B, H, L) : 0;
+}
+
+hipError_t scan_split_launch(const ScanArgs& a, bool bf16_io, int len, void* ws, hipStream_t st) {
   const int nseg = (a.L + len - 1) / len;
   const long bhs = (long)a.B * a.H * nseg;
   Carries loc, in;
@@ -217,7 +281,9 @@ hipError_t scan_split_launch(const ScanArgs& a, bool bf16_io, void* ws, hipStrea
 }
 
 hipError_t scan_split_state_launch(const ScanArgs& a, bool bf16_io, void* ws, hipStream_t st) {
-  const int len = seg_len_for(a.B, a.H, a.L);
+  const int len = scan_split_len(bf16_io, a.B, a.L, a.H, a.N, a.P, a.R, 64,
+                                 scan_split_ws_bytes(bf16_io, a.B, a.L, a.H, a.N, a.P, a.R, 64));
+  if (len == 0) return scan_state_launch(a, bf16_io, st);
   const int nseg = (a.L + len - 1) / len;
   const long bhs = (long)a.B * a.H * nseg;
   Carries loc, in;

@@ -200,7 +200,7 @@ class Mamba3Layer:
         if in_place:
             pre(None, None)
             y = torch.empty(B, L, nh, hd, device=dev, dtype=dt)
-            ws_bytes = lib.m3_chunk_scan_ws_bytes(B, L, nh, N, hd, R, self.chunk_size, io)
+            ws_bytes = lib.m3_scan_split_plan_bytes(B, L, nh, N, hd, R, self.chunk_size, io)
             ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
             args = (_ptr(Q), _ptr(K), _ptr(proj), self.d_in_proj, _ptr(ADT), _ptr(DT), _ptr(Trap), _ptr(Ang),
                     _ptr(pp["C_bias"]), _ptr(pp["B_bias"]), _ptr(pp["D"]), _ptr(y), B, L, nh, N, hd, R,

@@ -136,7 +136,7 @@ def _launch(p, dims, chunk_size, out, init=None, fin=None, seq_split=True):
     tail = (B, L, H, HQ, N, P, R, int(chunk_size), io)
     ip = tuple(_ptr(t) for t in init) if init is not None else (None,) * 4
     fp = tuple(_ptr(t) for t in fin) if fin is not None else (None,) * 4
-    ws_bytes = lib.m3_chunk_scan_ws_bytes(B, L, H, N, P, R, int(chunk_size), io) if seq_split else 0
+    ws_bytes = lib.m3_scan_split_plan_bytes(B, L, H, N, P, R, int(chunk_size), io) if seq_split else 0
     if ws_bytes:
         # few (batch, head) pairs: the sequence is split across compute units; the
         # workspace lives for this call only (torch's caching allocator, same stream)
@@ -193,7 +193,7 @@ def _forward_train(args, chunk_size, seq_split):
         _launch(p, (B, L, H, HQ, N, P, R), chunk_size, out, seq_split=seq_split)
         return (out[0] if unbatched else out), None
     saved = torch.empty(nbytes, dtype=torch.uint8, device=p["V"].device)
-    ws_bytes = lib.m3_chunk_scan_ws_bytes(B, L, H, N, P, R, int(chunk_size), io) if seq_split else 0
+    ws_bytes = lib.m3_scan_split_plan_bytes(B, L, H, N, P, R, int(chunk_size), io) if seq_split else 0
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=p["V"].device)
     rc = lib.m3_chunk_scan_fwd_train(
         _ptr(p["Q"]), _ptr(p["K"]), _ptr(p["V"]), _ptr(p["ADT"]), _ptr(p["DT"]), _ptr(p["Trap"]),
@@ -377,7 +377,7 @@ def _shared_forward(args, chunk_size, seq_split, train=False, cdt=None):
     if out.numel():
         lib = _lib.load()
         io = _IO[p["V"].dtype]
-        ws_bytes = lib.m3_chunk_scan_ws_bytes(B, L, H, N, P, R, int(chunk_size), io) if seq_split else 0
+        ws_bytes = lib.m3_scan_split_plan_bytes(B, L, H, N, P, R, int(chunk_size), io) if seq_split else 0
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=p["V"].device)
         common = (_ptr(p["Q"]), _ptr(p["K"]), _ptr(p["V"]), _ptr(p["ADT"]), _ptr(p["DT"]), _ptr(p["Trap"]),
                   _ptr(p["Q_bias"]), _ptr(p["K_bias"]), _ptr(p["Angles"]), _ptr(p["D"]), _ptr(p["Z"]), _ptr(out),
