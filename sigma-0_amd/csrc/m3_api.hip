@@ -583,6 +583,41 @@ int m3_layer_decode_step(const void* proj, const float* dt_bias, const float* B_
 
 }  // extern "C"
 
+extern "C" {
+
+int m3_step_rows_max(int d_model, int d_inner, int d_in_proj) {
+  if (d_inner != 2 * d_model || !m3::step_gemm_supported(0, d_model, d_in_proj)) return 0;
+  // A whole captured step against the route of library products and single kernels (us):
+  // d_model 256, 8 blocks: 32 rows 164 / 307, 256 rows 393 / 639, 512 rows 602 / 703;
+  // 512, 8 blocks: 64 rows 301 / 442, 256 rows 672 / 747, 384 rows 893 / 926, 512 rows 1118 /
+  // 1124; 768, 12 blocks: 32 rows 437 / 580, 64 rows 630 / 762, 128 rows 928 / 1013, 192 rows
+  // 1253 / 1191; 1024, 8 blocks: 32 rows 404 / 494, 96 rows 692 / 719, 128 rows 862 / 823:
+  // beyond, the products are no longer latency and the library's larger tiles win.
+  return d_model > 768 ? 96 : d_model > 512 ? 128 : d_model > 256 ? 384 : 512;
+}
+
+int m3_step_gemm(int mode, const void* x, const void* wt, void* out, const float* scale, const float* bias,
+                 const void* b2, const float* skip, int M, int K, int N, float eps, void* stream) {
+  if (mode < 0 || mode > 3)
+    return fail(M3_E_ARG, "mode must be 0 (in_proj), 1 (out_proj), 2 (gate) or 3 (gelu and gate), got %d", mode);
+  if (M < 0 || K <= 0 || N <= 0) return fail(M3_E_ARG, "non-positive dimension (M=%d K=%d N=%d)", M, K, N);
+  if (!m3::step_gemm_supported(mode, K, N) || (mode >= 2 && K != N))
+    return fail(M3_E_UNSUPPORTED, "no step kernel for mode %d with K=%d N=%d", mode, K, N);
+  if (M == 0) {
+    g_err[0] = '\0';
+    return M3_OK;
+  }
+  if (!x || !wt || !out || (mode < 2 && !scale) || (mode == 0 && !bias) || (mode >= 2 && (!b2 || !skip)))
+    return fail(M3_E_ARG, "NULL required pointer");
+  const void* vec_ptrs[] = {x, wt, out, scale, bias, b2, skip};
+  for (const void* p : vec_ptrs)
+    if (!aligned16(p)) return fail(M3_E_ALIGN, "the step's operands must be 16-byte aligned");
+  m3::StepGemmArgs a{x, wt, out, scale, bias, b2, skip, M, K, N, eps};
+  return check_launch(m3::step_gemm_launch(mode, a, reinterpret_cast<hipStream_t>(stream)), "step gemm");
+}
+
+}  // extern "C"
+
 namespace {
 // The in-place layout of the layer's scan entry points: projection rows exactly
 // 2HP + 2N + 3H + R wide (the layout m3_layer_pre reads) and a multiple of 16 bytes;

@@ -260,6 +260,20 @@ struct DecodeArgs {
   float A_floor = 0.0f, eps = 0.0f;
 };
 
+// The generation step's Dense layers with their norms, gelu and gate (m3_step.hip), bf16:
+// out (M, N) = epilogue(prologue(x (M, K)) W).  mode 0 in_proj: x float32, LayerNorm
+// (scale, bias), wt = W (K, N); 1 out_proj: x bf16, RMSNorm (scale), wt = W (K, N), out
+// gelu; 2 gate (K = N): x bf16 (g), wt = W^T (N, K), b2 (N,) bf16, out float32 = skip + g
+// sigmoid(g W + b2); 3: the same with x the pre-gelu values, g = gelu(x).
+struct StepGemmArgs {
+  const void* x; const void* wt; void* out;
+  const float* scale; const float* bias; const void* b2; const float* skip;
+  int M, K, N;
+  float eps;
+};
+bool step_gemm_supported(int mode, int K, int N);
+hipError_t step_gemm_launch(int mode, const StepGemmArgs& a, hipStream_t st);
+
 bool decode_supported(int N, int P, int R);
 hipError_t decode_step_launch(const DecodeArgs& a, bool in_bf16, bool out_bf16, hipStream_t st);
 
@@ -268,4 +282,11 @@ hipError_t decode_step_launch(const DecodeArgs& a, bool in_bf16, bool out_bf16, 
 // Workspace bytes for the split that the library would choose itself (0: none), for the
 // bundled host wrappers, which pass a workspace of this size where the public contract
 // (m3_chunk_scan_ws_bytes) promises a smaller or no split.
-extern "C" size_t m3_scan_split_plan_bytes(int B, int L, int H, int N, int P, int R, int chunk_size, int io_dtype);
+extern "C" {
+size_t m3_scan_split_plan_bytes(int B, int L, int H, int N, int P, int R, int chunk_size, int io_dtype);
+// The generation step's fused Dense layers (m3::StepGemmArgs), for the bundled host
+// wrapper: the largest batch they are used for (0: never, for these sizes), and the call.
+int m3_step_rows_max(int d_model, int d_inner, int d_in_proj);
+int m3_step_gemm(int mode, const void* x, const void* wt, void* out, const float* scale, const float* bias,
+                 const void* b2, const float* skip, int M, int K, int N, float eps, void* stream);
+}

@@ -50,8 +50,11 @@ _SIGS = {
     "m3_chunk_scan_fwd": ([_P] * 12 + [_I] * 9 + [_P], _I),
     "m3_chunk_scan_fwd_carry": ([_P] * 20 + [_I] * 9 + [_P], _I),
     "m3_chunk_scan_ws_bytes": ([_I] * 8, ctypes.c_size_t),
-    # not part of the public ABI: the workspace of the split the library itself prefers
+    # not part of the public ABI: the workspace of the split the library itself prefers,
+    # and the generation step's fused Dense layers
     "m3_scan_split_plan_bytes": ([_I] * 8, ctypes.c_size_t),
+    "m3_step_rows_max": ([_I] * 3, _I),
+    "m3_step_gemm": ([_I] + [_P] * 7 + [_I] * 3 + [ctypes.c_float, _P], _I),
     "m3_chunk_scan_fwd_ws": ([_P] * 20 + [_I] * 9 + [_P, ctypes.c_size_t, _P], _I),
     "m3_chunk_scan_fwd_noalloc": ([_P] * 20 + [_I] * 9 + [_P], _I),
     "m3_chunk_scan_bwd_ws_bytes": ([_I] * 9, ctypes.c_size_t),

@@ -101,31 +101,47 @@ class Mamba3Layer:
         the token and the decode update in one launch: B and C shared over heads, trap
         through the sigmoid as the reference's recurrent path applies it),
         m3_layer_post and the out_proj GEMM."""
-        from .decode import recurrent_angle_mode, recurrent_diagonal_mode
-        from .ops import mamba3_contraction_precision_mode
         Bn = x_t.shape[0]
-        dt, dev = self.dtype, x_t.device
+        dt = self.dtype
+        self._check_carry(carry, Bn)
+        proj = torch.matmul(x_t.to(dt).reshape(Bn, 1, self.d_model), self.w_in).contiguous()
+        y = self._decode(proj, carry)
+        return self._project(y).reshape(Bn, self.d_model), carry
+
+    def _project(self, y: torch.Tensor) -> torch.Tensor:
+        """The output norm and out_proj of step's y (B, 1, d_inner)."""
+        yn = torch.empty_like(y)
+        _lib.check(_lib.load().m3_layer_post(_ptr(y), _ptr(self.params["out_norm"]), _ptr(yn), y.shape[0], 1,
+                                             self.d_inner, self.eps, _IO[self.dtype], _stream(y)), "m3_layer_post")
+        return torch.matmul(yn, self.w_out)
+
+    def _check_carry(self, carry, Bn: int) -> None:
+        """step's carry: float32, contiguous, in place."""
         nh, hd, N, R = self.nh, self.hd, self.N, self.R
-        lib, io, pp = _lib.load(), _IO[dt], self.params
         theta, ssm, kprev, vprev = carry
         for name, t, shape in (("theta", theta, (Bn, nh, R)), ("ssm", ssm, (Bn, nh, hd, N)),
                                ("k", kprev, (Bn, nh, N)), ("v", vprev, (Bn, nh, hd))):
             if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and tuple(t.shape) == shape):
                 raise ValueError(f"carry {name} must be a contiguous float32 device tensor of shape {shape} "
                                  "(it is updated in place)")
+
+    def _decode(self, proj: torch.Tensor, carry) -> torch.Tensor:
+        """m3_layer_decode_step on the tokens' in_proj rows (B, ..., d_in_proj): y (B, 1,
+        d_inner), the carry updated in place."""
+        from .decode import recurrent_angle_mode, recurrent_diagonal_mode
+        from .ops import mamba3_contraction_precision_mode
+        Bn, pp = proj.shape[0], self.params
+        theta, ssm, kprev, vprev = carry
         mamba3_contraction_precision_mode()     # the reference's decode reads it too (mamba3.py:545)
         angle, diag = recurrent_angle_mode(), recurrent_diagonal_mode()
-        proj = torch.matmul(x_t.to(dt).reshape(Bn, 1, self.d_model), self.w_in).contiguous()
-        y = torch.empty(Bn, 1, self.d_inner, device=dev, dtype=dt)
-        _lib.check(lib.m3_layer_decode_step(
+        y = torch.empty(Bn, 1, self.d_inner, device=proj.device, dtype=self.dtype)
+        _lib.check(_lib.load().m3_layer_decode_step(
             _ptr(proj), _ptr(pp["dt_bias"]), _ptr(pp["B_norm"]), _ptr(pp["C_norm"]), _ptr(pp["B_bias"]),
             _ptr(pp["C_bias"]), _ptr(pp["D"]), _ptr(theta), _ptr(ssm), _ptr(kprev), _ptr(vprev), _ptr(y),
-            Bn, nh, hd, N, R, self.A_floor, self.eps, io, 1 if angle == "wrapped" else 0,
-            1 if diag == "legacy_double" else 0, _stream(proj)), "m3_layer_decode_step")
-        yn = torch.empty(Bn, 1, self.d_inner, device=dev, dtype=dt)
-        _lib.check(lib.m3_layer_post(_ptr(y), _ptr(pp["out_norm"]), _ptr(yn), Bn, 1, self.d_inner, self.eps, io,
-                                     _stream(y)), "m3_layer_post")
-        return torch.matmul(yn, self.w_out).reshape(Bn, self.d_model), carry
+            Bn, self.nh, self.hd, self.N, self.R, self.A_floor, self.eps, _IO[self.dtype],
+            1 if angle == "wrapped" else 0, 1 if diag == "legacy_double" else 0, _stream(proj)),
+            "m3_layer_decode_step")
+        return y
 
     def train_forward(self, x: torch.Tensor) -> torch.Tensor:
         """forward, differentiable: gradients flow to x and to the parameter tensors the

@@ -44,6 +44,14 @@ from .ops import _IO, _ptr, _stream
 ACTIVATIONS = ("gelu", "full_glu", "half_glu1", "half_glu2")
 _ACT = dict(gelu=_lib.M3_ACT_GELU, full_glu=_lib.M3_ACT_FULL_GLU, half_glu1=_lib.M3_ACT_HALF_GLU1,
             half_glu2=_lib.M3_ACT_HALF_GLU2)
+# The fewest rows that the generation step's fused Dense layers take.  They accumulate over
+# the contraction in one order, which is the library's too from here up (in_proj and gate;
+# the out_proj up to 1024 inputs), so that the step's results stay bit for bit those of its
+# products.  Below, and for longer out_projs, the library splits the contraction: about 2
+# outputs in 10000 then round the other way, and over 12 blocks single carry entries move by
+# as much as their own size, so the library's products stay there (at one row the fused
+# route took 289 us where they take 476, d_model 768).
+_STEP_ROWS_MIN = 32
 
 
 class Mamba3Stack:
@@ -64,6 +72,16 @@ class Mamba3Stack:
                 b[n + "_w"] = lp[n + "_w"].to(dtype).t().contiguous()     # flax (in, out) -> F.linear (out, in)
                 b[n + "_b"] = lp[n + "_b"].to(dtype)
             self.blocks.append(b)
+        # The generation step's fused Dense layers (m3_step_gemm) run for batches from
+        # _STEP_ROWS_MIN up to step_rows_max (0: none, for other blocks and for parameters
+        # that are not 16-byte aligned).
+        self.step_rows_max = 0
+        if dtype == torch.bfloat16 and prenorm and activation == "half_glu1" and self.blocks and all(
+                t.data_ptr() % 16 == 0 for b in self.blocks for t in (b["ln_scale"], b["ln_bias"], b["out2_w"],
+                                                                      b["out2_b"], b["mixer"].params["out_norm"],
+                                                                      b["mixer"].w_in, b["mixer"].w_out)):
+            m = self.blocks[0]["mixer"]
+            self.step_rows_max = _lib.load().m3_step_rows_max(d_model, m.d_inner, m.d_in_proj)
         self.decoder_w = self.decoder_b = None
         self._dec_w3 = self._dec_w3b = None
         if "decoder_w" in params:
@@ -168,6 +186,8 @@ class Mamba3Stack:
         every block's mixer through its decode step (Mamba3Layer.step), the carries
         in ``state`` updated in place."""
         Bn = ids_t.shape[0]
+        if _STEP_ROWS_MIN <= Bn <= self.step_rows_max:
+            return self._head(self._step_fused(ids_t, state)), state
 
         def step_mixer(i):
             def run(t):
@@ -176,6 +196,34 @@ class Mamba3Stack:
             return run
         x = self.forward(ids_t.reshape(Bn, 1), mixers=[step_mixer(i) for i in range(len(self.blocks))])
         return self._head(x)[:, 0], state
+
+    def _step_fused(self, ids_t: torch.Tensor, state) -> torch.Tensor:
+        """step's features (B, d_model), per block: the in_proj Dense with the LayerNorm
+        before it, the decode update, the out_proj Dense between the output RMSNorm and the
+        gelu (d_inner > 1024: the norm, the library's product, and the gelu in the next
+        launch), and the gate's Dense with the gate and the residual add."""
+        lib = _lib.load()
+        D, Bn = self.d_model, ids_t.shape[0]
+        x = self.embed[ids_t.reshape(Bn)].contiguous()
+        st = _stream(x)
+        for i, b in enumerate(self.blocks):
+            m, carry = b["mixer"], state[i]
+            m._check_carry(carry, Bn)
+            proj = torch.empty(Bn, m.d_in_proj, device=x.device, dtype=self.dtype)
+            _lib.check(lib.m3_step_gemm(0, _ptr(x), _ptr(m.w_in), _ptr(proj), _ptr(b["ln_scale"]),
+                                        _ptr(b["ln_bias"]), None, None, Bn, D, m.d_in_proj, 1e-6, st), "m3_step_gemm")
+            y = m._decode(proj, carry)
+            if m.d_inner <= 1024:
+                g, gate = torch.empty(Bn, D, device=x.device, dtype=self.dtype), 2
+                _lib.check(lib.m3_step_gemm(1, _ptr(y), _ptr(m.w_out), _ptr(g), _ptr(m.params["out_norm"]), None, None,
+                                            None, Bn, m.d_inner, D, m.eps, st), "m3_step_gemm")
+            else:
+                g, gate = m._project(y), 3
+            out = torch.empty_like(x)
+            _lib.check(lib.m3_step_gemm(gate, _ptr(g), _ptr(b["out2_w"]), _ptr(out), None, None, _ptr(b["out2_b"]),
+                                        _ptr(x), Bn, D, D, 0.0, st), "m3_step_gemm")
+            x = out
+        return x
 
     __call__ = forward
 
@@ -307,7 +355,8 @@ class StepGraph:
     decode and block kernels, the head) with no host work between them.  It returns
     the log-probabilities (B, vocab) in the graph's output buffer, which the next call
     overwrites, and advances the carries of ``state`` in place, as step does.  The
-    decode mode knobs (MAMBA3_RECURRENT_*) are read once, at capture.  Nothing in the
+    decode mode knobs (MAMBA3_RECURRENT_*) are read once, at capture.  The graph reads the
+    stack's weights where they lie, so the stack must be kept as long.  Nothing in the
     step records a memset node: the library has none, and its buffers are written
     whole by their kernels."""
 
