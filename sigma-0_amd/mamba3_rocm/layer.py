@@ -34,7 +34,7 @@ from typing import Dict
 import torch
 
 from . import _lib
-from .ops import (_IO, _ptr, _stream, mamba3_siso_hip_carry, mamba3_ssd_chunked_shared_hip,
+from .ops import (_final_carry, _IO, _ptr, _stream, mamba3_siso_hip_carry, mamba3_ssd_chunked_shared_hip,
                   mamba3_ssd_chunked_shared_hip_bwd, mamba3_ssd_chunked_shared_hip_fwd_train, new_carry,
                   pallas_compute_dtype)
 
@@ -200,7 +200,7 @@ class Mamba3Layer:
                 for t, s_, n in zip(init, shapes, ("theta", "ssm", "k", "v")):
                     if tuple(t.shape) != s_:
                         raise ValueError(f"carry {n} must be {s_}, got {tuple(t.shape)}")
-            carry = new_carry(B, nh, N, hd, R, dev)
+            carry = _final_carry(B, L, nh, N, hd, R, dev)
         sbytes = 0
         if keep and in_place:
             # in place in training: the saved-state pair must exist for the shape (a

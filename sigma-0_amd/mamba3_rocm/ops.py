@@ -303,6 +303,17 @@ def new_carry(B: int, H: int, N: int, P: int, R: int, device) -> Tuple[torch.Ten
             torch.zeros(B, H, N, **z), torch.zeros(B, H, P, **z))
 
 
+def _final_carry(B: int, L: int, H: int, N: int, P: int, R: int, device) -> Tuple[torch.Tensor, ...]:
+    """A prefill's final carry.  Every scan kernel writes all of it, so it isn't cleared first
+    (four launches: 49 -> 35 us for 613 tokens of 24 heads in bf16), unless nothing is
+    launched."""
+    if not (B and L and H and P):
+        return new_carry(B, H, N, P, R, device)
+    z = dict(device=device, dtype=torch.float32)
+    return (torch.empty(B, H, R, **z), torch.empty(B, H, P, N, **z),
+            torch.empty(B, H, N, **z), torch.empty(B, H, P, **z))
+
+
 def mamba3_siso_hip_carry(Q, K, V, ADT, DT, Trap, Q_bias, K_bias, Angles, D=None, Z=None,
                           chunk_size: int = 64, initial_carry=None, seq_split: bool = True):
     """Prefill that also consumes and returns the recurrent carry, so decode can
@@ -313,7 +324,7 @@ def mamba3_siso_hip_carry(Q, K, V, ADT, DT, Trap, Q_bias, K_bias, Angles, D=None
     _req(not unbatched, "mamba3_siso_hip_carry takes batched (B, L, ...) inputs")
     B, L, H, HQ, N, P, R = dims
     out = torch.empty_like(p["V"])
-    fin = new_carry(B, H, N, P, R, p["V"].device)
+    fin = _final_carry(B, L, H, N, P, R, p["V"].device)
     init = None
     if initial_carry is not None:
         init = tuple(_f32(t) for t in initial_carry)
